@@ -94,3 +94,15 @@ def test_offsets_on_nodes_and_half_cells(order):
 def test_large_courant_number(order):
     """moves of up to 0.9 cells"""
     _check(order, (24, 18), 2000, c=0.9)
+
+
+@pytest.mark.parametrize("tile", [(8, 8, 1), (16, 8, 1), (16, 16, 1)])
+def test_every_move_leaves_the_window(tile):
+    """order 3, nearly every particle crosses a cell boundary in y, in several
+    passes: more moves than the list of a pass has room for (a quarter of its
+    particles), so rows are added both from the list and at once"""
+    def place(prt, base, rng):
+        up = rng.random(prt.shape[1]) < 0.5
+        prt[1] = np.floor(prt[1]) + np.where(up, 0.95, 0.05)
+        prt[4] = np.where(up, 1.5, -1.5)
+    _check(3, (24, 16), 6000, tile, place=place)
