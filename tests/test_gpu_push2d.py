@@ -106,3 +106,35 @@ def test_every_move_leaves_the_window(tile):
         prt[1] = np.floor(prt[1]) + np.where(up, 0.95, 0.05)
         prt[4] = np.where(up, 1.5, -1.5)
     _check(3, (24, 16), 6000, tile, place=place)
+
+
+@pytest.mark.parametrize("order", [1, 2, 3])
+def test_a_particle_that_is_not_a_number_stays_one(order):
+    """a NaN momentum gives NaN positions, not a number inside the grid, on
+    this push and the next, and leaves the other particles alone"""
+    import tmpg
+    nx, ny, n = 24, 18, 1500
+    p = dict(c=0.45, corr=1.025, c_omp=4.0, gamma0=0.5, ppc0=4.0, me=1.0, mi=16.0)
+    f, pi, pe = random_state(2, order, nx, ny, 1, n, seed=7)
+    cfg = orc.make_cfg(2, order, nx, ny, 1)
+    fields = orc.fill_from_interior(cfg, f, np.float32)[:6]
+    bad = (3, 777, n - 1)
+    out = []
+    for nan in (False, True):
+        if nan:
+            for q, s in zip(bad, (1.0, -1.0, 1.0)):
+                pi[3 + q % 3, q] = np.copysign(np.float32(np.nan), np.float32(s))
+        ctx = make_context(tmpg, 2, order, nx, ny, 1, p)
+        ctx.set_fields(fields)
+        ctx.set_particles(0, pi)
+        ctx.set_particles(1, pe)
+        ctx.push_deposit()
+        ctx.push_deposit()
+        out.append([sorted_by_id(*ctx.get_particles(s, with_ids=True)) for s in (0, 1)])
+        ctx.close()
+    (a0, a1), (b0, b1) = out
+    good = np.ones(n, bool)
+    good[list(bad)] = False
+    np.testing.assert_array_equal(a1, b1)
+    np.testing.assert_array_equal(a0[:, good], b0[:, good])
+    assert np.isnan(b0[:2, ~good]).all() and np.isnan(b0[3:6, ~good]).all()
