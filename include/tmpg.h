@@ -60,9 +60,11 @@ typedef struct tmpg_config {
     float   q[2];         /* charge per macro-particle: qi, qe */
     float   mass[2];      /* mi, me after normalisation (energy diagnostics) */
     int64_t capacity[2];  /* particle capacity per species (0: sized at first load) */
-    int32_t tile[3];      /* cell tile for the sorted push (0: default, 8x8x4 in
-                             3D (zigzag 8x8x2 or 8x4x2); in 2D 8x8, or up to 16x16 for a sparse plasma
-                             on a large grid) */
+    int32_t tile[3];      /* cell tile for the sorted push (all 0: default, 8x8x4
+                             in 3D (zigzag 8x8x2 or 8x4x2); in 2D 8x8, or up to
+                             16x16 for a sparse plasma on a large grid.  Axes
+                             left 0 beside an explicit one: 8x8x4 in 3D, in 2D
+                             16 wide and 16 rows, 8 on a small grid) */
     int32_t sort_every;   /* tmpg_step sorts each tile's particles by cell every
                              this many steps where its push reads them in
                              stored order (0: every 4 where that pays, in 3D
