@@ -67,9 +67,10 @@ typedef struct tmpg_config {
                              16 wide and 16 rows, 8 on a small grid) */
     int32_t sort_every;   /* tmpg_step sorts each tile's particles by cell every
                              this many steps where its push reads them in
-                             stored order (0: every 4 where that pays, in 3D
-                             for orders 3 and, without TMPG_Q_GATHER2, 2;
-                             negative: never) */
+                             stored order (0: every 4 where the push that runs
+                             gains from it, in 3D for the default tiles' order 3
+                             and, without TMPG_Q_GATHER2, 2, and other tiles'
+                             order 2; negative: never) */
     int32_t highorder;    /* nonzero: 4th-order field solver (<algorithm>
                              highorder; advance_b_halfstep_42 and
                              advance_e_fullstep_42, code/fields.F90:1039-1361) */

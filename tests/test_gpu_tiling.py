@@ -27,3 +27,52 @@ def test_partly_explicit_tiles(dim, shape, tile, scheme, fits):
     ctx = make_context(tmpg, dim, 1, *shape, P, tile=tile, scheme=scheme)
     assert np.isfinite(ctx.get_fields()).all()
     ctx.close()
+
+
+def _cells(ctx, dim, shape, species=0):
+    """cell coordinates of a species' particles in the library's order"""
+    h, hz = ctx.ng // 2, ctx.ngz // 2
+    p = ctx.get_particles(species)
+    lo = (h + 1, h + 1, hz + 1)
+    return [np.floor(p[a]).astype(np.int64) - lo[a] if a < dim else np.zeros(p.shape[1], np.int64) for a in range(3)]
+
+
+def _tile_ids(c, shape, tile):
+    nt = [-(-shape[a] // tile[a]) for a in range(3)]
+    t = [c[a] // tile[a] for a in range(3)]
+    return t[0] + nt[0] * (t[1] + nt[1] * t[2])
+
+
+def _load(ctx, dim, shape, n, seed, species=(0, 1)):
+    """n particles per species at rest, away from the cells' faces"""
+    h, hz = ctx.ng // 2, ctx.ngz // 2
+    for s in species:
+        rng = np.random.default_rng(seed + s)
+        p = np.zeros((7, n), np.float32)
+        for a, lo in enumerate((h + 1, h + 1, hz + 1)):
+            p[a] = lo + rng.integers(0, shape[a] if a < dim else 1, n) + 0.25 + 0.5 * rng.random(n)
+        p[6] = 1.0
+        ctx.set_particles(s, p)
+
+
+@pytest.mark.parametrize("dim,order,compat,tile,sorts", [
+    (3, 3, 7, (0, 0, 0), True), (3, 2, 0, (0, 0, 0), True), (3, 2, 7, (0, 0, 0), False), (3, 1, 7, (0, 0, 0), False),
+    (3, 3, 7, (8, 8, 8), False), (3, 2, 7, (8, 8, 2), True), (3, 2, 0, (8, 8, 2), True), (3, 1, 7, (8, 8, 2), False),
+    (2, 3, 7, (32, 8, 0), False), (2, 2, 7, (12, 12, 0), False),
+])
+def test_default_sort_goes_with_the_kernel(dim, order, compat, tile, sorts):
+    """the default sorts (before the fourth step) only where the push that
+    runs gains from it: the order within the tiles tells"""
+    import tmpg
+    shape = (16, 16, 8) if dim == 3 else (48, 24, 1)
+    ctx = make_context(tmpg, dim, order, *shape, P, compat=compat, tile=tile, track_ids=False)
+    _load(ctx, dim, shape, 12000, 11)
+    ctx.step(4)
+    c = _cells(ctx, dim, shape)
+    ctx.close()
+    size = [t or d for t, d in zip(tile, (8, 8, 4))] if dim == 3 else [tile[0], tile[1], 1]
+    t = _tile_ids(c, shape, size)
+    local = sum((c[a] % size[a]) * m for a, m in zip(range(3), (1, size[0], size[0] * size[1])))
+    same = t[1:] == t[:-1]
+    rising = np.mean(np.diff(local)[same] >= 0)
+    assert (rising > 0.9) == sorts and (rising < 0.6) != sorts

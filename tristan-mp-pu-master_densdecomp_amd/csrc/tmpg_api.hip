@@ -232,17 +232,6 @@ int tmpg_create(const tmpg_config* cfg, tmpg_ctx** out)
     ctx->cfg = *cfg;
     ctx->cfg.nz = nz;
     ctx->zz = cfg->scheme == TMPG_SCHEME_ZIGZAG;
-    // Sorted order pays where the 3D gather reads 64 nodes (orders 3 and 2
-    // without the reference's loop range): fewer LDS bank conflicts.  Particle
-    // phase without and with the sort, 96^3 cells: order 3 at 4 per cell and
-    // species 783, 758 us, at 16 2824, 2768; order 2 (64 nodes) 694, 701 and
-    // 2276, 2187.  With 8 nodes it costs more than it saves: order 1 640, 661
-    // and 1537, 1707; order 2 596, 625 and 1732, 1934.  Where the push adds to
-    // LDS particle by particle (2D tiles of a sparse plasma, zigzag),
-    // neighbouring lanes then add to the same words: 1024^2 cells, order 2, 2
-    // per cell 171, 198; zigzag, 80x64x48 cells, 8 per cell 173, 203.
-    const bool nodes64 = cfg->order == 3 || (cfg->order == 2 && !(cfg->compat & TMPG_Q_GATHER2));
-    ctx->sort_every = cfg->sort_every != 0 ? cfg->sort_every : cfg->dim == 3 && !ctx->zz && nodes64 ? 4 : -1;
     ctx->g.dim = cfg->dim;
     ctx->g.nx = cfg->nx;
     ctx->g.ny = cfg->ny;
@@ -740,6 +729,7 @@ int tmpg_step(tmpg_ctx* ctx, int nsteps)
             if (!rc) rc = particles_check(ctx);
             if (rc) break;
         }
+        const int sort_every = particles_sort_every(ctx);
         // code/tristanmainloop.F90:117-242 with the ghost fills and the
         // current fold absorbed into periodic indexing, reset_currents moved
         // before the push and add_current fused into the E update
@@ -754,7 +744,7 @@ int tmpg_step(tmpg_ctx* ctx, int nsteps)
         }
         rc = fields_bhalf(ctx, &first);
         mark(ctx, ST_PARTICLES);
-        if (!rc && ctx->sort_every > 0 && !particles_push_sorts(ctx) && ++ctx->steps_since_sort >= ctx->sort_every) {
+        if (!rc && sort_every > 0 && ++ctx->steps_since_sort >= sort_every) {
             ctx->steps_since_sort = 0;
             rc = particles_sort_tiles(ctx);
         }

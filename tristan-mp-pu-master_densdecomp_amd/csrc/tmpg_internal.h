@@ -154,7 +154,6 @@ struct tmpg_ctx {
     unsigned stamp_done = 0;       // boundaries stamped in the step under way
     bool stamping = false;         // inside tmpg_step
     int prof_steps = 0;            // steps summed in stamps
-    int sort_every = 4;                 // tmpg_step sorts each tile's particles by cell every this many steps
     int ncu = 256;                      // compute units of the context's device
     int steps_since_sort = 0;
     float* pin = nullptr;               // pinned pieces of the grid getters, with an event for each
@@ -225,8 +224,8 @@ int particles_load_uniform(tmpg_ctx* ctx, int s, int ppc, float drift, float the
 // apply fn to every live particle slot: kernels over the tiled layout use this
 int particles_check(tmpg_ctx* ctx);
 int particles_sort_tiles(tmpg_ctx* ctx);
-// the fused push orders the particles by cell itself: no sort between steps
-bool particles_push_sorts(const tmpg_ctx* ctx);
+// steps between tmpg_step's sorts of each tile's particles by cell; negative: none
+int particles_sort_every(const tmpg_ctx* ctx);
 int diag_energies(tmpg_ctx* ctx, double out[4]);
 int diag_rho(tmpg_ctx* ctx, double* rho_dev);
 int diag_continuity(tmpg_ctx* ctx, double* maxres, double* rhonorm);
