@@ -3,7 +3,7 @@ tiles fit a CU's LDS."""
 import numpy as np
 import pytest
 
-from gpu_util import make_context
+from gpu_util import make_context, periodic_diff, random_state, rel, sorted_by_id
 
 pytestmark = pytest.mark.gpu
 P = dict(c=0.45, corr=1.025, c_omp=4.0, gamma0=0.5, ppc0=4.0, me=1.0, mi=16.0)
@@ -76,3 +76,31 @@ def test_default_sort_goes_with_the_kernel(dim, order, compat, tile, sorts):
     same = t[1:] == t[:-1]
     rising = np.mean(np.diff(local)[same] >= 0)
     assert (rising > 0.9) == sorts and (rising < 0.6) != sorts
+
+
+@pytest.mark.parametrize("order,tile,ppc", [(1, (12, 12, 1), 6), (2, (32, 8, 1), 14), (3, (12, 12, 1), 3)])
+def test_sorted_run_matches_unsorted_2d(order, tile, ppc):
+    """tiles whose push reads the particles in stored order: sorted before every
+    step and never, they hold the same particles and fields up to the order of
+    the currents' additions (the bars of the sort's other tests)"""
+    import orc
+    import tmpg
+    nx, ny = 48, 32
+    f, pi, pe = random_state(2, order, nx, ny, 1, ppc * nx * ny, seed=60 + order, emax=0.02, bmax=0.05, umax=0.8)
+    full = orc.fill_from_interior(orc.make_cfg(2, order, nx, ny, 1), f, np.float32)[:6]
+    out = []
+    for sort_every in (1, -1):
+        ctx = make_context(tmpg, 2, order, nx, ny, 1, P, sort_every=sort_every, tile=tile)
+        ctx.set_fields(full)
+        ctx.set_particles(0, pi)
+        ctx.set_particles(1, pe)
+        ctx.step(6)
+        out.append(([sorted_by_id(*ctx.get_particles(s, with_ids=True)) for s in (0, 1)], ctx.get_fields()))
+        ctx.close()
+    (ps, fs), (pu, fu) = out
+    for s in (0, 1):
+        for r, n in ((0, nx), (1, ny)):
+            assert np.abs(periodic_diff(ps[s][r], pu[s][r], 0, n)).max() < 1e-4
+        assert rel(ps[s][3:6], pu[s][3:6]) < 1e-6
+    for q in range(6):
+        assert rel(fs[q], fu[q]) < 1e-5
