@@ -116,3 +116,16 @@ def test_crowded_cell(order, npart):
         prt[3:6] = 0.05 * rng.standard_normal((3, prt.shape[1]))
         prt[3] += 1.0
     _check(order, (16, 8, 8), npart, place=place)
+
+
+def test_one_dense_tile_among_sparse_ones():
+    """order 3 with a mean below the records of a pass, so the single-pass
+    kernel runs, and one tile of 4200 particles: its waves beyond the record
+    space give their slots back and deposit at once, crossers among them"""
+    def place(prt, base, rng):
+        first = rng.random(prt.shape[1]) < 0.47
+        prt[0] = base + np.where(first, (prt[0] - base) % 8, prt[0] - base)
+        m = rng.random(prt.shape[1]) < 0.5
+        prt[1] = np.where(m, np.floor(prt[1]) + 0.95, prt[1])
+        prt[4] = np.where(m, 1.5, prt[4])
+    _check(3, (32, 8, 4), 3500, place=place)
