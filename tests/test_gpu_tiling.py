@@ -104,3 +104,31 @@ def test_sorted_run_matches_unsorted_2d(order, tile, ppc):
         assert rel(ps[s][3:6], pu[s][3:6]) < 1e-6
     for q in range(6):
         assert rel(fs[q], fu[q]) < 1e-5
+
+
+def _tile(ctx, shape):
+    """the finest of the 2D default tiles that the particles run by (but for
+    single ones whose rounded position lies across a face)"""
+    c = _cells(ctx, 2, shape)
+    for tile in ((8, 8, 1), (16, 8, 1), (16, 16, 1)):
+        if np.mean(np.diff(_tile_ids(c, shape, tile)) < 0) < 1e-3:
+            return tile
+    return None
+
+
+@pytest.mark.parametrize("n,order,ppc,c,tile", [
+    (384, 2, 8, 0.6, (16, 16, 1)), (384, 2, 8, 0.45, (8, 8, 1)),           # a push without register sums
+    (128, 2, 8, 0.6, (8, 8, 1)),
+    (736, 1, 6, 0.45, (16, 16, 1)), (736, 1, 7, 0.45, (8, 8, 1)),          # eight tiles per CU
+    (736, 2, 5, 0.45, (16, 16, 1)), (736, 2, 6, 0.45, (8, 8, 1)),
+    (736, 3, 4, 0.45, (16, 8, 1)), (736, 3, 5, 0.45, (8, 8, 1)),
+    (384, 1, 3, 0.45, (16, 16, 1)), (384, 1, 4, 0.45, (8, 8, 1)),          # two
+    (384, 2, 2, 0.45, (16, 16, 1)), (384, 2, 3, 0.45, (8, 8, 1)),
+])
+def test_default_tiles_2d(n, order, ppc, c, tile):
+    import tmpg
+    ctx = make_context(tmpg, 2, order, n, n, 1, dict(P, c=c), track_ids=False)
+    for s in (0, 1):
+        ctx.load_uniform(s, ppc, 0.0, 0.01, 3 + s)
+    assert _tile(ctx, (n, n, 1)) == tile
+    ctx.close()
