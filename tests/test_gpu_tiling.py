@@ -132,3 +132,37 @@ def test_default_tiles_2d(n, order, ppc, c, tile):
         ctx.load_uniform(s, ppc, 0.0, 0.01, 3 + s)
     assert _tile(ctx, (n, n, 1)) == tile
     ctx.close()
+
+
+@pytest.mark.parametrize("loads,tile", [
+    (((0, 2), (1, 14)), (8, 8, 1)), (((1, 14), (0, 2)), (8, 8, 1)),
+    (((0, 4),), (16, 16, 1)), (((1, 6), (0, 0)), (16, 16, 1)), (((0, 1), (1, 1), (1, 8)), (8, 8, 1)),
+])
+@pytest.mark.parametrize("push", ["step", "push_deposit", "move"])
+def test_tiles_go_with_all_particles(loads, tile, push):
+    """the tiles of a run are those of its whole density, in whatever order and
+    parts the species come"""
+    import tmpg
+    n = 384
+    ctx = make_context(tmpg, 2, 1, n, n, 1, P, track_ids=False)
+    for k, (s, ppc) in enumerate(loads):
+        if ppc:
+            ctx.load_uniform(s, ppc, 0.0, 0.01, 3 + k)
+    before = [ctx.get_particles(s) for s in (0, 1)]
+    if push == "step":
+        ctx.step(1)
+    else:
+        getattr(ctx, push)()
+    shape = (n, n, 1)
+    for s in (0, 1):
+        if before[s].shape[1]:
+            c = _cells(ctx, 2, shape, s)
+            assert np.mean(np.diff(_tile_ids(c, shape, tile)) < 0) < 1e-3
+            finer = (8, 8, 1) if tile[0] == 16 else (8, 4, 1)
+            assert np.mean(np.diff(_tile_ids(c, shape, finer)) < 0) > 0.01
+        after = ctx.get_particles(s)
+        assert after.shape == before[s].shape
+        if push != "step":
+            u0, u1 = (np.sort(x[3]) for x in (before[s], after))
+            assert rel(u1, u0) < 1e-5 or u0.size == 0
+    ctx.close()

@@ -626,12 +626,14 @@ static int pre_push(tmpg_ctx* ctx)
 int tmpg_move(tmpg_ctx* ctx)
 {
     if (!valid_ctx(ctx)) return TMPG_EINVAL;
+    int rc = particles_retile(ctx);
+    if (rc) return rc;
     for (auto& s : ctx->sp)
         if (s.n > 0) {
-            int rc = alloc_split_scratch(ctx, s);
+            rc = alloc_split_scratch(ctx, s);
             if (rc) return rc;
         }
-    int rc = pre_push(ctx);
+    rc = pre_push(ctx);
     if (rc) return rc;
     rc = particles_push(ctx, 1);
     if (rc == TMPG_OK) ctx->move_pending = true;
@@ -650,7 +652,8 @@ int tmpg_deposit(tmpg_ctx* ctx)
 int tmpg_push_deposit(tmpg_ctx* ctx)
 {
     if (!valid_ctx(ctx)) return TMPG_EINVAL;
-    int rc = pre_push(ctx);
+    int rc = particles_retile(ctx);
+    if (!rc) rc = pre_push(ctx);
     if (rc) return rc;
     ctx->move_pending = false;
     return particles_push(ctx, 0);
@@ -727,6 +730,11 @@ int tmpg_step(tmpg_ctx* ctx, int nsteps)
             ctx->steps_since_check = 0;
             rc = flush_stamps(ctx);
             if (!rc) rc = particles_check(ctx);
+            if (rc) break;
+        }
+        if (ctx->tiling_due) {
+            rc = flush_stamps(ctx);
+            if (!rc) rc = particles_retile(ctx);
             if (rc) break;
         }
         const int sort_every = particles_sort_every(ctx);

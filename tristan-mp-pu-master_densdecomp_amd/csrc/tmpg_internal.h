@@ -156,6 +156,7 @@ struct tmpg_ctx {
     int prof_steps = 0;            // steps summed in stamps
     int ncu = 256;                      // compute units of the context's device
     int steps_since_sort = 0;
+    bool tiling_due = false;            // particles came since the tiling was last compared
     float* pin = nullptr;               // pinned pieces of the grid getters, with an event for each
     int64_t pin_cap = 0;                // (floats)
     hipEvent_t pin_ev[8] = {};
@@ -214,6 +215,9 @@ int particles_bin(tmpg_ctx* ctx, int s, const PBuf& flat, int64_t n, bool has_ch
 // compact copy of all live particles of species s into flat (device), n out
 int particles_flatten(tmpg_ctx* ctx, int s, PBuf& flat, int64_t* n);
 int particles_rebalance(tmpg_ctx* ctx, int s);
+// before a push: both species binned anew where the default tiling of what has
+// been loaded differs from the one they were binned by
+int particles_retile(tmpg_ctx* ctx);
 // the tiling of a configuration whose two species together hold per_cell
 // particles per cell (0: not known)
 Tiling default_tiling(const tmpg_config& cfg, int ncu, double per_cell);
