@@ -134,14 +134,12 @@ __device__ __forceinline__ void place(const float* v, int base, int first, float
     }
 }
 
-// Shape profile of one axis of a cell-summed record on a fixed node window:
-// S = old weights, dS = new - old.  profile6: nodes [-2,3] (x, cell
-// crossings included); profile4: nodes [-1,2] (y, z: the record's move keeps
-// the support inside the window).  Order 3 writes the pieces straight into
-// their slots: the old piece is the particle's own cell (m0 = 0), the new
-// one is m1 = floor(o + d) in {-1, 0, 1}, and a crossing splits dS at the
-// knot K = max(m0, m1) exactly as axis_deposit does.  Other orders go
-// through axis_deposit and place the window.
+// Shape profile of one axis of a cell-summed record on nodes [-2,3] (cell
+// crossings included): S = old weights, dS = new - old.  Order 3 writes the
+// pieces straight into their slots: the old piece is the particle's own cell
+// (m0 = 0), the new one is m1 = floor(o + d) in {-1, 0, 1}, and a crossing
+// splits dS at the knot K = max(m0, m1) exactly as axis_deposit does.  Other
+// orders go through axis_deposit and place the window.
 template <int ORD>
 __device__ __forceinline__ void profile6(float o, float d, float* S6, float* dS6)
 {
@@ -172,21 +170,6 @@ __device__ __forceinline__ void profile6(float o, float d, float* S6, float* dS6
         const int b = axis_deposit<ORD>(o, d, S1, dS);
         place<W, 6>(S1, b, -2, S6);
         place<W, 6>(dS, b, -2, dS6);
-    }
-}
-
-template <int ORD>
-__device__ __forceinline__ void profile4(float o, float d, float* S4, float* dS4)
-{
-    if constexpr (ORD == 3) {
-        Piece<3>::w(o, S4);
-        Piece<3>::dw(o, o + d, d, dS4);
-    } else {
-        constexpr int W = Win<ORD>::W;
-        float S1[W], dS[W];
-        const int b = axis_deposit<ORD>(o, d, S1, dS);
-        place<W, 4>(S1, b, -1, S4);
-        place<W, 4>(dS, b, -1, dS4);
     }
 }
 
@@ -243,7 +226,8 @@ __device__ __forceinline__ void window4(float o, float d, float* S, float* dS)
         dS[2] = (p0 ? t0[1] : t0[2]) + (p1 ? t1[1] : t1[2]);
         dS[3] = (p0 ? t0[2] : 0.0f) + (p1 ? t1[2] : 0.0f);
     } else {
-        profile4<3>(o, d, S, dS);
+        Piece<3>::w(o, S);
+        Piece<3>::dw(o, o + d, d, dS);
     }
 }
 

@@ -296,8 +296,6 @@ int tmpg_create(const tmpg_config* cfg, tmpg_ctx** out)
     for (int q = 0; q < NF && e == hipSuccess; ++q) e = hipMemsetAsync(ctx->f[q], 0, ctx->g.n * sizeof(float), ctx->stream);
     if (e == hipSuccess) e = hipMemsetAsync(ctx->flags, 0, 16 * sizeof(int32_t), ctx->stream);
     if (e == hipSuccess) e = hipMemsetAsync(ctx->stamps, 0, 16 * sizeof(unsigned long long), ctx->stream);
-    for (auto& ev : ctx->ev)
-        if (e == hipSuccess) e = hipEventCreate(&ev);
     if (e != hipSuccess) {
         g_create_err = std::string("tmpg_create: ") + hipGetErrorString(e);
         tmpg_destroy(ctx);
@@ -343,8 +341,6 @@ int tmpg_destroy(tmpg_ctx* ctx)
     dfree(ctx->red);
     dfree(ctx->flags);
     for (auto& s : ctx->sp) free_species(s);
-    for (auto& ev : ctx->ev)
-        if (ev) (void)hipEventDestroy(ev);
     if (ctx->stamps) (void)hipFree(ctx->stamps);
     if (ctx->hostcnt) (void)hipHostFree(ctx->hostcnt);
     if (ctx->pin) (void)hipHostFree(ctx->pin);

@@ -145,7 +145,6 @@ struct tmpg_ctx {
     bool cnt_pending = false;
     uint32_t cnt_seq = 0;
     int steps_since_check = 0;
-    hipEvent_t ev[8] = {};
     // per-phase timing of tmpg_step: the first kernel of a phase adds the
     // device's clock to the sum of that boundary, so the phases' times are
     // differences of the sums, and no event goes into the stream
